@@ -85,6 +85,14 @@ constexpr int kPiecesPerGroup = CSRSPMM_PIECES_PER_GROUP;
 #define CSRSPMM_SWEEP_WPE 8
 #endif
 
+// The least waves per SIMD that the one-chunk kernels of row units are
+// compiled for; build-time tunable.  Their segment blocks would take 80
+// registers (6 waves) without it: 8192 x 4096 x 256 with 410 per row 127 us
+// against 118.
+#ifndef CSRSPMM_ROWS_WPE
+#define CSRSPMM_ROWS_WPE 8
+#endif
+
 // Split rows summed in the main launch (Problem::seg_fuse); 0: always the
 // combine launch.
 #ifndef CSRSPMM_SEG_FUSE
@@ -680,9 +688,8 @@ __device__ __forceinline__ void store_partial(float* dst, float v) {
 // the same order.  Byte offsets fit 31 bits (launch_rowgroup_all fuses only
 // when the whole partial buffer does).
 constexpr int kCpolSc1 = 16;  // the sc1 cache-policy bit of buffer instructions
-template <int NG>
-__device__ __forceinline__ f4 sum_strided_coh(__amdgpu_buffer_rsrc_t rsrc, int c, int n, int q, long long ldp,
-                                              bool cv) {
+__device__ __forceinline__ f4 sum_strided_coh(__amdgpu_buffer_rsrc_t rsrc, int c, int n, int q, int ng,
+                                              long long ldp, bool cv) {
   f4 acc = Vec<4>::zero();
   if (!cv) return acc;
   auto part = [&](int k) -> f4 {
@@ -690,29 +697,33 @@ __device__ __forceinline__ f4 sum_strided_coh(__amdgpu_buffer_rsrc_t rsrc, int c
     return __builtin_bit_cast(f4, __builtin_amdgcn_raw_buffer_load_b128(rsrc, off, 0, kCpolSc1));
   };
   int k = q;
-  for (; k + 3 * NG < n; k += 4 * NG) {
+  for (; k + 3 * ng < n; k += 4 * ng) {
     f4 a[4];
 #pragma unroll
-    for (int u = 0; u < 4; ++u) a[u] = part(k + u * NG);
+    for (int u = 0; u < 4; ++u) a[u] = part(k + u * ng);
 #pragma unroll
     for (int u = 0; u < 4; ++u) acc = add_v(acc, a[u]);
   }
-  for (; k < n; k += NG) acc = add_v(acc, part(k));
+  for (; k < n; k += ng) acc = add_v(acc, part(k));
   return acc;
 }
 
 // The split rows that this wave's groups counted last (lanes in `pend`, each
 // holding row, segments n and first position x0), one after another with
 // the whole wave, in the combine's lane layout and order (combine_kernel's
-// slot scan: GC lanes a float4 chunk, 64 / GC groups adding strided
+// slot scan: gc lanes a float4 chunk, 64 / gc groups adding strided
 // partials, then the xor tree), so a fused row is bit for bit the combined
-// one.
-template <int VEC, int GC>
+// one.  gc, as launch_combine picks it from N, is a run-time value here: four
+// compiled copies, one per gc, cost the kernel registers.
+template <int VEC>
 __device__ __forceinline__ void fused_rows(const Problem& p, unsigned long long pend, int row, int n, int x0) {
-  constexpr int P = 64 / GC;
+  const int chunks = (p.N + 3) / 4;
+  const int gshift = chunks <= 8 ? 3 : chunks <= 16 ? 4 : chunks <= 32 ? 5 : 6;
+  const int gc = 1 << gshift;
   const int lane = lane_id();
-  const int q = lane / GC;
-  const int gl = lane & (GC - 1);
+  const int q = lane >> gshift;
+  const int gl = lane & (gc - 1);
+#pragma unroll 1
   while (pend) {
     const int l = __ffsll((long long)pend) - 1;
     pend &= pend - 1;
@@ -722,19 +733,39 @@ __device__ __forceinline__ void fused_rows(const Problem& p, unsigned long long 
     const __amdgpu_buffer_rsrc_t rsrc =
         __builtin_amdgcn_make_buffer_rsrc(base, (short)0, (int)((long long)nn * p.ldp * 4), 0x00020000);
     float* crow = p.C + (long long)r * p.ldc;
-    for (int c0 = 0; c0 < p.N; c0 += GC * 4) {
+#pragma unroll 1
+    for (int c0 = 0; c0 < p.N; c0 += gc * 4) {
       const int c = c0 + gl * 4;
       const bool cv = c < p.N;
-      const f4 acc = wave_group_sum<GC>(sum_strided_coh<P>(rsrc, c, nn, q, p.ldp, cv));
+      f4 acc = sum_strided_coh(rsrc, c, nn, q, 64 >> gshift, p.ldp, cv);
+#pragma unroll 1
+      for (int off = gc; off < 64; off <<= 1) {
+        const int src = (lane ^ off) << 2;
+        auto other = [&](float v) {
+          return __builtin_bit_cast(float, __builtin_amdgcn_ds_bpermute(src, __builtin_bit_cast(int, v)));
+        };
+        const f4 o = f4{other(acc.x), other(acc.y), other(acc.z), other(acc.w)};
+        acc = add_v(acc, o);
+      }
       if (q == 0 && cv) store_cols4<VEC>(p, crow + c, c, acc);
     }
   }
 }
 
+// Rows of block b of a launch with row units: block b runs on XCD b mod
+// kXcds, and rows whose length follows the bits of their index (R-MAT: 0.76
+// of the edges per zero bit) would load the XCDs as unevenly, so the low
+// digit of b is xored with its higher ones.  A permutation of every aligned
+// group of kXcds blocks (the grid holds whole groups).
+__device__ __forceinline__ int row_block(int b) {
+  int x = b ^ (b >> 3) ^ (b >> 6) ^ (b >> 9) ^ (b >> 12) ^ (b >> 15) ^ (b >> 18);
+  return (b & ~(kXcds - 1)) | (x & (kXcds - 1));
+}
+
 // One block's share of the main launch, over the columns [c_lo, c_hi):
 // block bid < seg_blocks takes long-row segment slots, the others merge
 // blocks of short rows (or, without a plan, rows).
-template <int VEC, int G, int T, int U, bool LDS, bool BUF, int SU, bool SWEEP, bool FUSE>
+template <int VEC, int G, int T, int U, bool LDS, bool BUF, int SU, bool SWEEP, bool FUSE, bool ROWS>
 __device__ __forceinline__ void rowgroup_block(const Problem& p, int bid, int seg_blocks, int c_lo,
                                                int c_hi, int gl, int gbase, int gid, int2* stage,
                                                int* sweep_bnd) {
@@ -747,19 +778,15 @@ __device__ __forceinline__ void rowgroup_block(const Problem& p, int bid, int se
     // counts last (over every column slice) notes the row in fuse_row, and
     // once the gathers are done its wave sums the rows its groups noted.
     constexpr int US = SU > U ? (SU < G ? SU : G) : U;
-    auto slot = [&](int s, int& fuse_row, int& fuse_n, int& fuse_x0) {
-      const int2 si = p.seg_info[s];
-      if (si.x < 0 || si.x >= p.M) return;  // unused slot
-      const int rs = p.rowptr[si.x];
-      const int re = p.rowptr[si.x + 1];
+    // Segment k of row `row` [rs, re), of slot s.
+    auto segment = [&](int s, int srow, int k, int rs, int re, int& fuse_row, int& fuse_n, int& fuse_x0) {
       const int len = re - rs;
-      if (len >= kPanelMinLen && is_panelized(p, rs)) return;  // summed by the pieces kernel
       const int nseg = seg_count(p, len);
-      const int start = rs + seg_begin(len, nseg, si.y);
-      const int end = rs + seg_begin(len, nseg, si.y + 1);
-      // partial si.y of the row (si.y < the segments plan_kernel counted
-      // from the clamped row range, so this stays inside the buffer)
-      float* prow = p.partials + ((long long)(clamp_nnz(rs, p.nnz) >> p.seg_shift) + si.y) * p.ldp;
+      const int start = rs + seg_begin(len, nseg, k);
+      const int end = rs + seg_begin(len, nseg, k + 1);
+      // partial k of the row (k < the segments plan_kernel counted from the
+      // clamped row range, so this stays inside the buffer)
+      float* prow = p.partials + ((long long)(clamp_nnz(rs, p.nnz) >> p.seg_shift) + k) * p.ldp;
       for (int c0 = c_lo; c0 < c_hi; c0 += PW) {
         const Panel<VEC, G, T, BUF> pn(p, c0, gl, c_hi);
         VT acc[T];
@@ -771,7 +798,7 @@ __device__ __forceinline__ void rowgroup_block(const Problem& p, int bid, int se
                                               for (int t = 0; t < T; ++t) acc[t] = fma_v(v, b[t], acc[t]);
                                             });
         if (nseg == 1) {  // the whole row: epilogue and store here
-          store_row<VEC, T>(p, si.x, pn.col, pn.cval, acc);
+          store_row<VEC, T>(p, srow, pn.col, pn.cval, acc);
         } else if constexpr (FUSE) {
 #pragma unroll
           for (int t = 0; t < T; ++t) {
@@ -808,26 +835,61 @@ __device__ __forceinline__ void rowgroup_block(const Problem& p, int bid, int se
         }
       }
     };
+    auto slot = [&](int s, int& fuse_row, int& fuse_n, int& fuse_x0) {
+      const int2 si = p.seg_info[s];
+      if (si.x < 0 || si.x >= p.M) return;  // unused slot
+      const int rs = p.rowptr[si.x];
+      const int re = p.rowptr[si.x + 1];
+      if (re - rs >= kPanelMinLen && is_panelized(p, rs)) return;  // summed by the pieces kernel
+      segment(s, si.x, si.y, rs, re, fuse_row, fuse_n, fuse_x0);
+    };
+    // The rows that this wave's groups counted last, summed with the whole
+    // wave, one after another.
+    auto sum_fused = [&](int fuse_row, int fuse_n, int fuse_x0) {
+      const unsigned long long pend = __ballot(fuse_row >= 0 && gl == 0);
+      if (pend) fused_rows<VEC>(p, pend, fuse_row, fuse_n, fuse_x0);
+    };
     int fuse_row = -1, fuse_n = 0, fuse_x0 = 0;
-    if constexpr (FUSE) {
+    if constexpr (ROWS) {
+      // Each wave takes up to 64 slots, one per lane, nw apart (a row's
+      // neighbouring segments go to different waves), and its groups sum the
+      // segments of split rows among them; rows of one segment are row
+      // units.
+      const int nw = seg_blocks * kWaves;
+      const int per_wave = div_up(p.nslots, nw);
+      const int lane = lane_id();
+      const int s = bid * kWaves + gid / (64 / G) + lane * nw;
+      int2 si = make_int2(-1, 0);
+      int rs = 0, re = 0;
+      if (lane < per_wave && s < p.nslots) si = p.seg_info[s];
+      if (si.x >= 0 && si.x < p.M) {
+        rs = p.rowptr[si.x];
+        re = p.rowptr[si.x + 1];
+      }
+      unsigned long long todo = __ballot(seg_count(p, re - rs) >= 2);
+#pragma unroll 1
+      while (todo) {
+        // the wave's group i takes the i-th of the remaining slots
+        unsigned long long m = todo;
+        for (int i = 0; i < gbase / G; ++i) m &= m - 1;
+        const int l = m ? __ffsll((long long)m) - 1 : -1;
+#pragma unroll
+        for (int i = 0; i < 64 / G; ++i) todo &= todo - 1;
+        const int from = l < 0 ? 0 : l;
+        const int srow = __shfl(si.x, from);
+        const int k = __shfl(si.y, from);
+        const int a = __shfl(rs, from);
+        const int e = __shfl(re, from);
+        fuse_row = -1;
+        if (l >= 0) segment(bid * kWaves + gid / (64 / G) + l * nw, srow, k, a, e, fuse_row, fuse_n, fuse_x0);
+        if constexpr (FUSE) sum_fused(fuse_row, fuse_n, fuse_x0);
+      }
+    } else if constexpr (FUSE) {
       // one slot per group: a fused launch's segment blocks are not capped
       // (launch_rowgroup_all)
       const int s = bid * GPB + gid;
       if (s < p.nslots) slot(s, fuse_row, fuse_n, fuse_x0);
-      // the whole wave, its groups' rows one after another (GC as launch_combine picks it)
-      const unsigned long long pend = __ballot(fuse_row >= 0 && gl == 0);
-      if (pend) {
-        const int chunks = (p.N + 3) / 4;
-        if (chunks <= 8) {
-          fused_rows<VEC, 8>(p, pend, fuse_row, fuse_n, fuse_x0);
-        } else if (chunks <= 16) {
-          fused_rows<VEC, 16>(p, pend, fuse_row, fuse_n, fuse_x0);
-        } else if (chunks <= 32) {
-          fused_rows<VEC, 32>(p, pend, fuse_row, fuse_n, fuse_x0);
-        } else {
-          fused_rows<VEC, 64>(p, pend, fuse_row, fuse_n, fuse_x0);
-        }
-      }
+      sum_fused(fuse_row, fuse_n, fuse_x0);
     } else {
       for (int s = bid * GPB + gid; s < p.nslots; s += seg_blocks * GPB) slot(s, fuse_row, fuse_n, fuse_x0);
     }
@@ -845,7 +907,27 @@ __device__ __forceinline__ void rowgroup_block(const Problem& p, int bid, int se
                                    stage);
     return;
   }
-  if (p.plan) {
+  if constexpr (ROWS) {
+    // One row per group, summed whole; a split row's segments are summed by
+    // the segment blocks.
+    const int row = row_block(bid - seg_blocks) * GPB + gid;
+    if (row >= p.M) return;
+    const int start = p.rowptr[row];
+    const int end = p.rowptr[row + 1];
+    if (p.plan && seg_count(p, end - start) >= 2) return;
+    for (int c0 = c_lo; c0 < c_hi; c0 += PW) {
+      const Panel<VEC, G, T, BUF> pn(p, c0, gl, c_hi);
+      VT acc[T];
+#pragma unroll
+      for (int t = 0; t < T; ++t) acc[t] = Vec<VEC>::zero();
+      stream_nonzeros<VEC, G, T, U, LDS, BUF>(p, pn, start, end, gl, gbase, stage,
+                                         [&](int, float v, const VT(&b)[T]) {
+#pragma unroll
+                                           for (int t = 0; t < T; ++t) acc[t] = fma_v(v, b[t], acc[t]);
+                                         });
+      store_row<VEC, T>(p, row, pn.col, pn.cval, acc);
+    }
+  } else {
     // One merge block of short rows.
     if (unit >= p.nblocks) return;
     const int rs = max(0, p.block_start[unit]);
@@ -854,25 +936,6 @@ __device__ __forceinline__ void rowgroup_block(const Problem& p, int bid, int se
       const Panel<VEC, G, T, BUF> pn(p, c0, gl, c_hi);
       stream_rows<VEC, G, T, U, LDS, BUF>(p, pn, rs, re, gl, gbase, stage);
     }
-    return;
-  }
-
-  // No plan: one row per group, summed whole.
-  const int row = unit;
-  if (row >= p.M) return;
-  const int start = p.rowptr[row];
-  const int end = p.rowptr[row + 1];
-  for (int c0 = c_lo; c0 < c_hi; c0 += PW) {
-    const Panel<VEC, G, T, BUF> pn(p, c0, gl, c_hi);
-    VT acc[T];
-#pragma unroll
-    for (int t = 0; t < T; ++t) acc[t] = Vec<VEC>::zero();
-    stream_nonzeros<VEC, G, T, U, LDS, BUF>(p, pn, start, end, gl, gbase, stage,
-                                       [&](int, float v, const VT(&b)[T]) {
-#pragma unroll
-                                         for (int t = 0; t < T; ++t) acc[t] = fma_v(v, b[t], acc[t]);
-                                       });
-    store_row<VEC, T>(p, row, pn.col, pn.cval, acc);
   }
 }
 
@@ -929,8 +992,9 @@ __device__ __forceinline__ void interleave_roles(int b, int piece_blocks, int to
 // and the scalar N = 128 / 256 kernels 3-18% on the reference's sweep shapes.
 // FUSE: the segment blocks sum the split rows themselves (Problem::seg_fuse),
 // in instances of their own, so that the other kernels keep their registers.
-template <int VEC, int G, int T, int U, bool LDS, bool PIECES, int SU, bool BUF, bool SWEEP, bool FUSE = false>
-__global__ __launch_bounds__(kWaves * 64) __attribute__((amdgpu_waves_per_eu(SWEEP ? CSRSPMM_SWEEP_WPE : 1))) void rowgroup_kernel(Problem p, int piece_blocks,
+template <int VEC, int G, int T, int U, bool LDS, bool PIECES, int SU, bool BUF, bool SWEEP, bool FUSE = false,
+          bool ROWS = false>
+__global__ __launch_bounds__(kWaves * 64) __attribute__((amdgpu_waves_per_eu(SWEEP ? CSRSPMM_SWEEP_WPE : ROWS && T == 1 ? CSRSPMM_ROWS_WPE : 1))) void rowgroup_kernel(Problem p, int piece_blocks,
                                                                 int seg_blocks, int slice_blocks,
                                                                 int slice0) {
   constexpr int GPW = 64 / G;  // groups per wave
@@ -992,7 +1056,7 @@ __global__ __launch_bounds__(kWaves * 64) __attribute__((amdgpu_waves_per_eu(SWE
       bid = bid >= units ? bid - units : bid + seg_blocks;
     }
   }
-  rowgroup_block<VEC, G, T, U, LDS, BUF, SU, SWEEP, FUSE>(p, bid, seg_blocks, c_lo, c_hi, gl, gbase, gid, stage,
+  rowgroup_block<VEC, G, T, U, LDS, BUF, SU, SWEEP, FUSE, ROWS>(p, bid, seg_blocks, c_lo, c_hi, gl, gbase, gid, stage,
                                                      sweep_bnd);
 }
 
@@ -1145,7 +1209,7 @@ __global__ __launch_bounds__(256) void plan_kernel(Problem p) {
       const long long F = (long long)r + x0;
       const long long Fprev = r > 0 ? (long long)(r - 1) + clamp_nnz(p.rowptr[r - 1], p.nnz) : -1;
       b_lo = Fprev < 0 ? 0 : (int)((Fprev >> mshift) + 1);
-      b_hi = (int)min(F >> mshift, (long long)p.nblocks - 1);
+      b_hi = p.row_units ? b_lo - 1 : (int)min(F >> mshift, (long long)p.nblocks - 1);
       if (r == p.M) {
         p.block_start[p.nblocks] = p.M;
       } else {
@@ -1579,6 +1643,20 @@ void launch_combine(const Problem& p, hipStream_t s) {
   }
 }
 
+// Segment blocks of a launch with row units: at most kRowSegWaves waves, each
+// checking its share of the slots at once (up to 64 a wave), unless the rows
+// average a segment or more and most slots are used.  With a group a slot,
+// 8192 x 4096 x 256 with 410 per row (26,000 slots, none used) took 127 us
+// against 118.
+constexpr int kRowSegWaves = 4096;
+inline int row_seg_blocks(const Problem& p, int gpb) {
+  if (p.no_split) return 0;
+  int waves = div_up_host(p.nslots, gpb / kWaves);
+  const bool mostly_split = (long long)p.nnz >= ((long long)p.M << p.seg_shift);
+  if (!mostly_split && waves > kRowSegWaves) waves = std::max(kRowSegWaves, div_up_host(p.nslots, 64));
+  return div_up_host(waves, kWaves);
+}
+
 // SU: B-row gathers in flight per lane in the long-row segments (at least U).
 // BUF: B gathered through a buffer resource (buf_gathers_ok must hold).
 // SWEEP: the short rows of each slice in a band sweep (p.sweep_bands > 0).
@@ -1587,14 +1665,18 @@ template <int VEC, int G, int T, int U, bool LDS, int SU = CSRSPMM_SEG_UNROLL, b
           bool SWEEP = false>
 hipError_t launch_rg(const Problem& p, hipStream_t s) {
   constexpr int GPB = kWaves * (64 / G);
-  const int units = SWEEP ? div_up_host(p.M, kSweepRows) : p.plan ? p.nblocks : p.M;
-  const int unit_blocks = div_up_host(units, GPB);
+  // Row units: no plan, or a plan whose short rows are not merged (row_units).
+  const bool rows = !SWEEP && (!p.plan || p.row_units);
+  const int units = SWEEP ? div_up_host(p.M, kSweepRows) : rows ? p.M : p.nblocks;
+  const int unit_blocks = rows ? kXcds * div_up_host(div_up_host(units, GPB), kXcds) : div_up_host(units, GPB);
   // With XCD shares the segments run in share_kernel, launched before each
   // main launch over the same slices, and the main launch has no segment
   // blocks.
   const bool shares = p.plan && p.nslots > 0 && p.shares;
-  const int seg_blocks =
-      (p.plan && p.nslots > 0 && !shares) ? std::min(kSegBlocksMax, div_up_host(p.nslots, GPB)) : 0;
+  int seg_blocks = 0;
+  if (p.plan && p.nslots > 0 && !shares) {
+    seg_blocks = rows ? row_seg_blocks(p, GPB) : std::min(kSegBlocksMax, div_up_host(p.nslots, GPB));
+  }
   const int share_blocks =
       shares ? kXcds * div_up_host(div_up_host(p.nslots, std::min(G, CSRSPMM_SHARE_LANES)), GPB) : 0;
   constexpr int US = SU > U ? (SU < G ? SU : G) : U;
@@ -1634,6 +1716,18 @@ hipError_t launch_rg(const Problem& p, hipStream_t s) {
       hipLaunchKernelGGL((rowgroup_kernel<VEC, G, T, U, LDS, kCanPanel, SU, BUF, false>), dim3((unsigned)blocks),
                          dim3(kWaves * 64), pad_lds, s, p, piece_blocks, seg_blocks, slice_blocks,
                          s0);
+    } else if (rows) {
+      if constexpr (!SWEEP) {
+        if (p.seg_fuse) {
+          hipLaunchKernelGGL((rowgroup_kernel<VEC, G, T, U, LDS, false, U, BUF, false, true, true>),
+                             dim3((unsigned)blocks), dim3(kWaves * 64), pad_lds, s, p, 0, seg_blocks,
+                             slice_blocks, s0);
+        } else {
+          hipLaunchKernelGGL((rowgroup_kernel<VEC, G, T, U, LDS, false, U, BUF, false, false, true>),
+                             dim3((unsigned)blocks), dim3(kWaves * 64), pad_lds, s, p, 0, seg_blocks,
+                             slice_blocks, s0);
+        }
+      }
     } else if (p.seg_fuse) {
       hipLaunchKernelGGL((rowgroup_kernel<VEC, G, T, U, LDS, false, SU, BUF, SWEEP, true>), dim3((unsigned)blocks),
                          dim3(kWaves * 64), pad_lds, s, p, 0, seg_blocks, slice_blocks, s0);
@@ -1653,6 +1747,9 @@ static inline int pow2_ceil(int x) {
   return v;
 }
 
+// Group width of a float4 call covering n columns.
+static int vec4_group(int n) { return n >= 256 ? 64 : std::max(4, pow2_ceil(n / 4)); }
+
 // Unsliced float4 calls: the group width from N.
 // Unsliced float4 calls of up to 128 columns sweep too when B exceeds
 // CSRSPMM_SWEEP_UNSLICED_MB and the max_row_nnz hint rules out skewed rows
@@ -1669,19 +1766,11 @@ template <bool LDS, bool BUF>
 static hipError_t dispatch_vec4_cols(const Problem& p, hipStream_t s) {
   constexpr int SU = CSRSPMM_SEG_UNROLL;
   const int nv = (p.sw > 0 ? std::min(p.sw, p.N) : p.N) / 4;
-  const int G = nv >= 64 ? 64 : (pow2_ceil(nv) < 4 ? 4 : pow2_ceil(nv));
+  const int G = vec4_group(4 * nv);
   if constexpr (BUF) {
-    const long long mean4 = p.M > 0 ? 4LL * p.nnz / p.M : 0;
-    if ((G == 16 || G == 32) && p.dp.P == 0 && p.row_hint >= 0 &&
-        p.row_hint <= std::max<long long>(p.long_row, mean4) &&
-        (long long)p.K * p.N * 4 > ((long long)CSRSPMM_SWEEP_UNSLICED_MB << 20) &&
-        sweep_applies(p.plan, p.M, p.K, p.nnz, G * 4)) {
-      Problem q = p;
-      sweep_geometry(p.K, G * 4, q.sweep_shift, q.sweep_bands);
-      if (q.sweep_bands >= 2) {
-        if (G == 16) return launch_rg<4, 16, 1, kVec4U, LDS, CSRSPMM_SWEEP_SU, true, true>(q, s);
-        return launch_rg<4, 32, 1, kVec4U, LDS, CSRSPMM_SWEEP_SU, true, true>(q, s);
-      }
+    if (p.sweep_bands > 0) {
+      if (G == 16) return launch_rg<4, 16, 1, kVec4U, LDS, CSRSPMM_SWEEP_SU, true, true>(p, s);
+      return launch_rg<4, 32, 1, kVec4U, LDS, CSRSPMM_SWEEP_SU, true, true>(p, s);
     }
   }
   if (G < 64) {
@@ -1720,6 +1809,28 @@ static bool buf_gathers_ok(const Problem& p, int vec) {
   return (cols & (cols - 1)) == 0 && cols >= 4 * vec && (p.sw == 0 || p.N % p.sw == 0);
 }
 
+// Sets p.sweep_shift and p.sweep_bands when the main launch is a band sweep
+// (sweep_rows): of the short rows of each column slice, but for XCD slices,
+// which keep each band in one XCD's L2 without it, or of all N <= 128
+// columns.  The LDS-staged variant passes each chunk through its stage.
+static void set_sweep(Problem& p, int vec) {
+  p.sweep_shift = p.sweep_bands = 0;
+  if (vec != 4 || !p.plan || p.xslice || !buf_gathers_ok(p, 4)) return;
+  if (p.sw == kSliceWidth) {
+    if (sweep_applies(p.plan, p.M, p.K, p.nnz, p.sw)) sweep_geometry(p.K, p.sw, p.sweep_shift, p.sweep_bands);
+    return;
+  }
+  const int G = vec4_group(p.N);
+  const long long mean4 = p.M > 0 ? 4LL * p.nnz / p.M : 0;
+  if ((G != 16 && G != 32) || p.dp.P != 0 || p.row_hint < 0 ||
+      p.row_hint > std::max<long long>(p.long_row, mean4) ||
+      (long long)p.K * p.N * 4 <= ((long long)CSRSPMM_SWEEP_UNSLICED_MB << 20) ||
+      !sweep_applies(p.plan, p.M, p.K, p.nnz, G * 4))
+    return;
+  sweep_geometry(p.K, G * 4, p.sweep_shift, p.sweep_bands);
+  if (p.sweep_bands < 2) p.sweep_bands = 0;
+}
+
 // The kernel shape comes from the columns one block covers: a column slice,
 // or all N.
 //
@@ -1744,14 +1855,7 @@ static hipError_t dispatch_vec4(const Problem& p, hipStream_t s) {
   // configs within 1%.  Unsliced 16-lane calls keep 4 (XL at N = 64 lost 7%).
   static_assert(kSliceWidth == 64, "a slice's float4 chunks fill 16-lane groups");
   if (p.sw == kSliceWidth) {
-    // The short rows of each slice are swept band by band (sweep_rows); the
-    // LDS-staged variant passes each chunk through its stage.
-    // (XCD slices keep each band in one XCD's L2 without it.)
-    if (!p.xslice && sweep_applies(p.plan, p.M, p.K, p.nnz, p.sw) && buf_gathers_ok(p, 4)) {
-      Problem q = p;
-      sweep_geometry(p.K, p.sw, q.sweep_shift, q.sweep_bands);
-      return launch_rg<4, 16, 1, kVec4U, LDS, CSRSPMM_SWEEP_SU, true, true>(q, s);
-    }
+    if (p.sweep_bands > 0) return launch_rg<4, 16, 1, kVec4U, LDS, CSRSPMM_SWEEP_SU, true, true>(p, s);
     if (buf_gathers_ok(p, 4)) return launch_rg<4, 16, 1, kVec4U, LDS, 8, true>(p, s);
     return launch_rg<4, 16, 1, kVec4U, LDS, 8>(p, s);
   }
@@ -1817,6 +1921,35 @@ static hipError_t dispatch_main(const Problem& p, int vec, bool lds, hipStream_t
   return lds ? dispatch_vec1<true>(p, s) : dispatch_vec1<false>(p, s);
 }
 
+// Row units (Problem::row_units): each group sums one row whole, and only the
+// rows of two segments or more go to the segment blocks.  Merge blocks give
+// the groups of a wave equal items whatever the rows, but cut at every mblk
+// items: of rows longer than that some groups get none, rows above long_row
+// leave part of their segment slots' groups idle, and every nonzero is
+// checked against its row's end.  So long rows, and rows that the hint shows
+// to be about equal (at most 9/4 of the mean), take units; skewed short rows,
+// whose lengths differ within a wave, keep the merge blocks.  Measured on
+// MI355X per call, merge blocks -> row units: 4096^2 x 128 with 205 per row
+// 28.7 -> 23.6 us (WarpPerRowSmemFp4 41.6 -> 23.6), 8192 x 4096 x 256 with
+// 410 150 -> 118 and with 1229 (all of them split) 415 -> 402, 16384^2 x 128
+// with 82 42.8 -> 38.3, 16384^2 x 256 with 0-500 394 -> 251, 20000^2 x 512
+// with 100 317 -> 237; scalar columns, 30011 x 20021 x 47 with 0-300 95 ->
+// 72, 65536 x 16384 x 64 with 100 105 -> 78.  Below 64 per row: uniform rows
+// of 8 (131072 x 16384 x 128) 42.3 -> 35.2, of 24 (65536 x 8192 x 128) 46 ->
+// 39; scalar, of 48 (65536 x 16384 x 48) 47 -> 40, of 32 (x 64) 63.5 -> 61.8,
+// of 16 (x 48) 23 -> 26; but power-law rows (mean 16, 65536 x 16384 x 128) 62
+// -> 72 and R-MAT (32 per row, x 100) 137 -> 242.
+constexpr int kRowUnitMean = 64;
+constexpr int kRowUnitHintVec4 = 8;
+constexpr int kRowUnitHintScalar = 32;
+static bool row_units(const Problem& p, int vec) {
+  if (!p.plan || p.sweep_bands > 0 || p.shares || p.dp.P > 0 || p.npan > 0 || p.M <= 0) return false;
+  if ((long long)p.nnz >= (long long)kRowUnitMean * p.M) return true;
+  const int least = vec == 4 ? kRowUnitHintVec4 : kRowUnitHintScalar;
+  return p.row_hint >= 0 && (long long)p.nnz >= (long long)least * p.M &&
+         p.row_hint <= 9LL * p.nnz / (4LL * p.M);
+}
+
 static hipError_t launch_rowgroup_all(const Problem& p_in, int vec, bool lds, hipStream_t s) {
   // A per-call plan without column panels, XCD shares or stored panels sums
   // its split rows in the main launch (Problem::seg_fuse), when every slot
@@ -1829,11 +1962,15 @@ static hipError_t launch_rowgroup_all(const Problem& p_in, int vec, bool lds, hi
   // rows' sums one lane group at a time, with a load in flight, had cost
   // that call 58 us.
   Problem p = p_in;
+  set_sweep(p, vec);
+  p.row_units = row_units(p, vec);
   p.seg_fuse = CSRSPMM_SEG_FUSE && p.plan && !p.plan_ready && p.nslots > 0 && !p.no_split && !p.shares &&
                p.npan == 0 && p.dp.P == 0 && p.seg_cnt != nullptr &&
-               (long long)p.nslots <= (long long)kSegBlocksMax * kWaves &&
+               (p.row_units || (long long)p.nslots <= (long long)kSegBlocksMax * kWaves) &&
                (long long)(p.nnz >> p.seg_shift) * p.ldp * 4 < (1LL << 31);
-  if (p.plan && !p.plan_ready) hipLaunchKernelGGL(plan_kernel, dim3(plan_blocks(p)), dim3(256), 0, s, p);
+  // row units of a call without split rows need no tables
+  const bool tables = p.plan && !p.plan_ready && !(p.row_units && p.no_split);
+  if (tables) hipLaunchKernelGGL(plan_kernel, dim3(plan_blocks(p)), dim3(256), 0, s, p);
   hipError_t e;
   if (p.dp.P > 0 && !p.dp_ready) {
     e = launch_panel_schedule(p, s);

@@ -471,6 +471,10 @@ struct Problem {
   // slice) adds its partial rows, so no combine is launched.
   bool seg_fuse;
   int* seg_cnt;
+  // The main launch takes rows instead of merge blocks (row_units in
+  // rowgroup.hip): a row of fewer than two segments is summed whole by its
+  // own group, whatever its length.
+  bool row_units;
 };
 
 // XCD shares.  On a B far larger than the L2s, with no column panels (hot
