@@ -63,6 +63,11 @@ HIP_API = {
                                              _c_void_p, _c_void_p]),
     "csrspmm_dense2csr_fill_f32": (_c_int, [_c_int, _c_int, _c_void_p, _c_ll, _c_float, _c_void_p,
                                             _c_void_p, _c_void_p, _c_void_p]),
+    "csrspmm_dense2csr_scratch_bytes": (_c_size_t, [_c_int, _c_int]),
+    "csrspmm_dense2csr_count_f32_ex": (_c_int, [_c_int, _c_int, _c_void_p, _c_ll, _c_float, _c_void_p,
+                                                _c_void_p, _c_void_p, _c_size_t, _c_void_p]),
+    "csrspmm_dense2csr_fill_f32_ex": (_c_int, [_c_int, _c_int, _c_void_p, _c_ll, _c_float, _c_void_p,
+                                               _c_void_p, _c_void_p, _c_void_p, _c_size_t, _c_void_p]),
     "csrspmm_csr_max_row_nnz": (_c_int, [_c_int, _c_void_p, _c_void_p, _c_void_p]),
     "csrspmm_indices_i64_to_i32": (_c_int, [_c_void_p, _c_void_p, _c_ll, _c_void_p, _c_void_p]),
     "csrspmm_device_malloc": (_c_int, [ctypes.POINTER(_c_void_p), _c_size_t]),

@@ -267,7 +267,7 @@ hipStream_t stream_of(const Tensor& t) {
 }
 
 // Device dense -> CSR: (rowptr, colidx, values).  One host sync, to size
-// colidx/values from the count.
+// colidx/values from the count, which the scan writes to pinned host memory.
 std::vector<Tensor> dense_to_csr(Tensor D, double tol) {
   TORCH_CHECK(D.is_cuda(), "dense must be a CUDA tensor");
   TORCH_CHECK(D.dtype() == torch::kFloat32, "dense must be float32");
@@ -278,19 +278,32 @@ std::vector<Tensor> dense_to_csr(Tensor D, double tol) {
   const int M = static_cast<int>(D.size(0)), K = static_cast<int>(D.size(1));
   const long long ld = leading_dim(D, "dense");
   Tensor rowptr = torch::empty({M + 1}, D.options().dtype(torch::kInt32));
-  Tensor nnz = torch::empty({1}, D.options().dtype(torch::kInt64));
+  Tensor nnz = torch::empty({1}, torch::TensorOptions().dtype(torch::kInt64).pinned_memory(true));
+  // without room for the scratch the matrix is read twice
+  Tensor scratch;
+  size_t bytes = csrspmm_dense2csr_scratch_bytes(M, K);
+  if (bytes > 0) {
+    try {
+      scratch = torch::empty({static_cast<int64_t>(bytes)}, D.options().dtype(torch::kUInt8));
+    } catch (const c10::OutOfMemoryError&) {
+      bytes = 0;
+    }
+  }
+  void* sp = bytes > 0 ? scratch.data_ptr() : nullptr;
   hipStream_t s = stream_of(D);
   const float* d = D.numel() ? D.data_ptr<float>() : nullptr;
-  int st = csrspmm_dense2csr_count_f32(M, K, d, ld, static_cast<float>(tol), rowptr.data_ptr<int>(),
-                                       reinterpret_cast<long long*>(nnz.data_ptr<int64_t>()), s);
+  int st = csrspmm_dense2csr_count_f32_ex(M, K, d, ld, static_cast<float>(tol), rowptr.data_ptr<int>(),
+                                          reinterpret_cast<long long*>(nnz.data_ptr<int64_t>()), sp, bytes, s);
   TORCH_CHECK(st == 0, "dense_to_csr failed: ", csrspmm_status_string(st));
-  const int64_t n = nnz.item<int64_t>();
+  st = csrspmm_stream_synchronize(s);
+  TORCH_CHECK(st == 0, "dense_to_csr failed: ", csrspmm_status_string(st));
+  const int64_t n = *nnz.data_ptr<int64_t>();
   TORCH_CHECK(n <= INT32_MAX, "dense_to_csr: ", n, " nonzeros exceed int32");
   Tensor colidx = torch::empty({n}, D.options().dtype(torch::kInt32));
   Tensor vals = torch::empty({n}, D.options());
-  st = csrspmm_dense2csr_fill_f32(M, K, d, ld, static_cast<float>(tol), rowptr.data_ptr<int>(),
-                                  n ? colidx.data_ptr<int>() : nullptr,
-                                  n ? vals.data_ptr<float>() : nullptr, s);
+  st = csrspmm_dense2csr_fill_f32_ex(M, K, d, ld, static_cast<float>(tol), rowptr.data_ptr<int>(),
+                                     n ? colidx.data_ptr<int>() : nullptr,
+                                     n ? vals.data_ptr<float>() : nullptr, sp, bytes, s);
   TORCH_CHECK(st == 0, "dense_to_csr failed: ", csrspmm_status_string(st));
   return {rowptr, colidx, vals};
 }

@@ -334,7 +334,8 @@ int csrspmm_validate_csr(int M, int K, int nnz,
  * fabsf(v) > tol, so +-0 and NaN are dropped, in row-major order.  Two steps,
  * because the output size depends on the data:
  *  1. csrspmm_dense2csr_count_f32 writes rowptr[0..M] and the nonzero count
- *     as a 64-bit integer to *nnz_out (both device memory);
+ *     as a 64-bit integer to *nnz_out (both device memory, or host memory
+ *     that the device can write);
  *  2. after allocating colidx and vals for that count (it must fit int32),
  *     csrspmm_dense2csr_fill_f32 fills them.  Step 2 must see the same dense
  *     values, tol and rowptr as step 1.
@@ -343,6 +344,18 @@ int csrspmm_dense2csr_count_f32(int M, int K, const float* dense, long long ld, 
                                 int* rowptr, long long* nnz_out, void* stream);
 int csrspmm_dense2csr_fill_f32(int M, int K, const float* dense, long long ld, float tol,
                                const int* rowptr, int* colidx, float* vals, void* stream);
+/* The same two steps with a scratch of csrspmm_dense2csr_scratch_bytes(M, K)
+ * bytes (256-byte aligned device memory, passed unchanged from step 1 to
+ * step 2), in which step 1 keeps what step 2 needs of the matrix: it is read
+ * once, but for the parts of a row of which more than 3/8 are kept.  0 bytes
+ * (few columns, or a scratch beyond 8 GiB) or a NULL scratch: the steps above. */
+size_t csrspmm_dense2csr_scratch_bytes(int M, int K);
+int csrspmm_dense2csr_count_f32_ex(int M, int K, const float* dense, long long ld, float tol,
+                                   int* rowptr, long long* nnz_out, void* scratch,
+                                   size_t scratch_bytes, void* stream);
+int csrspmm_dense2csr_fill_f32_ex(int M, int K, const float* dense, long long ld, float tol,
+                                  const int* rowptr, int* colidx, float* vals,
+                                  const void* scratch, size_t scratch_bytes, void* stream);
 
 /* *max_out (device memory) = the longest row of rowptr[0..M]: the
  * max_row_nnz that the reference's dense2csr scans on the host
