@@ -557,6 +557,7 @@ int csrspmm_plan_spmm_f32(csrspmm_plan_t plan, int N, const float* B, long long 
     d.block_start = p->d_unit_start;
     d.nslots = 0;
     d.npan = 0;
+    d.pieces = true;
     d.rows_whole = true;  // pieces (at most kPieceMaxLen nonzeros) are summed whole
     d.no_split = true;
     e = launch_rowgroup(d, vec, lds, s);

@@ -711,15 +711,16 @@ __device__ __forceinline__ f4 sum_strided_coh(__amdgpu_buffer_rsrc_t rsrc, int c
 // The split rows that this wave's groups counted last (lanes in `pend`, each
 // holding row, segments n and first position x0), one after another with
 // the whole wave, in the combine's lane layout and order (combine_kernel's
-// slot scan: gc lanes a float4 chunk, 64 / gc groups adding strided
+// slot scan: GC lanes a float4 chunk, 64 / GC groups adding strided
 // partials, then the xor tree), so a fused row is bit for bit the combined
-// one.  gc, as launch_combine picks it from N, is a run-time value here: four
-// compiled copies, one per gc, cost the kernel registers.
-template <int VEC>
+// one.  GC as launch_combine picks it from N; 0: at run time, for the kernels
+// of row units, which four compiled copies would cost 48 registers (the copies
+// save the others 1 us on small split rows).
+template <int VEC, int GC>
 __device__ __forceinline__ void fused_rows(const Problem& p, unsigned long long pend, int row, int n, int x0) {
   const int chunks = (p.N + 3) / 4;
-  const int gshift = chunks <= 8 ? 3 : chunks <= 16 ? 4 : chunks <= 32 ? 5 : 6;
-  const int gc = 1 << gshift;
+  const int gc = GC > 0 ? GC : chunks <= 8 ? 8 : chunks <= 16 ? 16 : chunks <= 32 ? 32 : 64;
+  const int gshift = GC > 0 ? __builtin_ctz(GC > 0 ? GC : 1) : chunks <= 8 ? 3 : chunks <= 16 ? 4 : chunks <= 32 ? 5 : 6;
   const int lane = lane_id();
   const int q = lane >> gshift;
   const int gl = lane & (gc - 1);
@@ -738,14 +739,17 @@ __device__ __forceinline__ void fused_rows(const Problem& p, unsigned long long 
       const int c = c0 + gl * 4;
       const bool cv = c < p.N;
       f4 acc = sum_strided_coh(rsrc, c, nn, q, 64 >> gshift, p.ldp, cv);
+      if constexpr (GC > 0) {
+        acc = wave_group_sum<GC>(acc);
+      } else {
 #pragma unroll 1
-      for (int off = gc; off < 64; off <<= 1) {
-        const int src = (lane ^ off) << 2;
-        auto other = [&](float v) {
-          return __builtin_bit_cast(float, __builtin_amdgcn_ds_bpermute(src, __builtin_bit_cast(int, v)));
-        };
-        const f4 o = f4{other(acc.x), other(acc.y), other(acc.z), other(acc.w)};
-        acc = add_v(acc, o);
+        for (int off = gc; off < 64; off <<= 1) {
+          const int src = (lane ^ off) << 2;
+          auto other = [&](float v) {
+            return __builtin_bit_cast(float, __builtin_amdgcn_ds_bpermute(src, __builtin_bit_cast(int, v)));
+          };
+          acc = add_v(acc, f4{other(acc.x), other(acc.y), other(acc.z), other(acc.w)});
+        }
       }
       if (q == 0 && cv) store_cols4<VEC>(p, crow + c, c, acc);
     }
@@ -847,7 +851,21 @@ __device__ __forceinline__ void rowgroup_block(const Problem& p, int bid, int se
     // wave, one after another.
     auto sum_fused = [&](int fuse_row, int fuse_n, int fuse_x0) {
       const unsigned long long pend = __ballot(fuse_row >= 0 && gl == 0);
-      if (pend) fused_rows<VEC>(p, pend, fuse_row, fuse_n, fuse_x0);
+      if (!pend) return;
+      if constexpr (ROWS) {
+        fused_rows<VEC, 0>(p, pend, fuse_row, fuse_n, fuse_x0);
+      } else {
+        const int chunks = (p.N + 3) / 4;
+        if (chunks <= 8) {
+          fused_rows<VEC, 8>(p, pend, fuse_row, fuse_n, fuse_x0);
+        } else if (chunks <= 16) {
+          fused_rows<VEC, 16>(p, pend, fuse_row, fuse_n, fuse_x0);
+        } else if (chunks <= 32) {
+          fused_rows<VEC, 32>(p, pend, fuse_row, fuse_n, fuse_x0);
+        } else {
+          fused_rows<VEC, 64>(p, pend, fuse_row, fuse_n, fuse_x0);
+        }
+      }
     };
     int fuse_row = -1, fuse_n = 0, fuse_x0 = 0;
     if constexpr (ROWS) {
@@ -1939,15 +1957,28 @@ static hipError_t dispatch_main(const Problem& p, int vec, bool lds, hipStream_t
 // 39; scalar, of 48 (65536 x 16384 x 48) 47 -> 40, of 32 (x 64) 63.5 -> 61.8,
 // of 16 (x 48) 23 -> 26; but power-law rows (mean 16, 65536 x 16384 x 128) 62
 // -> 72 and R-MAT (32 per row, x 100) 137 -> 242.
+//
+// Where the typical row is split and the matrix is so small that the segments
+// are shortened, or has fewer than kRowUnitSplitRows rows, the scan costs the
+// segment blocks more than the rows gain, and the merge blocks' launch stays:
+// 2912 x 1061 x 64 with 302 per row 25.2 against 28.5 us, 1112 x 895 x 16
+// with 121 13.1 against 16.0, 1148 x 4292 x 256 with 1227 113 against 122.  So
+// it does for fewer than kRowUnitSliceRows rows a slice launched by itself,
+// whose few waves need the segments' deeper gathers: 5856 x 62064 x 220 with
+// 0-279 168 against 179.
 constexpr int kRowUnitMean = 64;
+constexpr int kRowUnitSplitRows = 2048;
+constexpr int kRowUnitSliceRows = 8192;
 constexpr int kRowUnitHintVec4 = 8;
 constexpr int kRowUnitHintScalar = 32;
 static bool row_units(const Problem& p, int vec) {
-  if (!p.plan || p.sweep_bands > 0 || p.shares || p.dp.P > 0 || p.npan > 0 || p.M <= 0) return false;
-  if ((long long)p.nnz >= (long long)kRowUnitMean * p.M) return true;
-  const int least = vec == 4 ? kRowUnitHintVec4 : kRowUnitHintScalar;
-  return p.row_hint >= 0 && (long long)p.nnz >= (long long)least * p.M &&
-         p.row_hint <= 9LL * p.nnz / (4LL * p.M);
+  if (!p.plan || p.sweep_bands > 0 || p.shares || p.dp.P > 0 || p.npan > 0 || p.pieces || p.M <= 0) return false;
+  const long long least = vec == 4 ? kRowUnitHintVec4 : kRowUnitHintScalar;
+  const bool equal = p.row_hint >= 0 && p.nnz >= least * p.M && p.row_hint <= 9LL * p.nnz / (4LL * p.M);
+  const bool split = !p.no_split && p.nnz >= (2LL * p.M << p.seg_shift) &&
+                     ((1 << p.seg_shift) < kSegLen || p.M < kRowUnitSplitRows);
+  const bool narrow = p.sw > 0 && p.slice_launch && p.M < kRowUnitSliceRows;
+  return (p.nnz >= (long long)kRowUnitMean * p.M || equal) && !split && !narrow;
 }
 
 static hipError_t launch_rowgroup_all(const Problem& p_in, int vec, bool lds, hipStream_t s) {

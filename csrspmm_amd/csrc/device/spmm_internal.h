@@ -475,6 +475,10 @@ struct Problem {
   // rowgroup.hip): a row of fewer than two segments is summed whole by its
   // own group, whatever its length.
   bool row_units;
+  // The rows are the pieces of a stored plan's panelized rows, whose merge
+  // blocks place them on the XCDs: they keep them (in row units 18 -> 29 us on
+  // power-law rows, 59534 x 44380 x 256).
+  bool pieces;
 };
 
 // XCD shares.  On a B far larger than the L2s, with no column panels (hot

@@ -42,6 +42,7 @@ def check(C, rp, ci, va, B, C0, alpha, beta, whole, what):
 CASES = [
     (1, 70000, 64, 66000, 66000, ()),                      # one row, all of it split
     (33, 4096, 128, 2000, 4000, ()),                       # every row split
+    (2101, 4096, 64, 600, 700, ()),                        # every row split, in row units
     (1003, 3000, 47, 0, 300, (0, 511, 512, 1002)),         # odd columns, no whole block
     (1003, 3000, 1, 0, 300, (5, 1002)),
     (2049, 2048, 8, 60, 140, (2048,)),
