@@ -70,6 +70,8 @@ HIP_API = {
                                                _c_void_p, _c_void_p, _c_void_p, _c_size_t, _c_void_p]),
     "csrspmm_csr_max_row_nnz": (_c_int, [_c_int, _c_void_p, _c_void_p, _c_void_p]),
     "csrspmm_indices_i64_to_i32": (_c_int, [_c_void_p, _c_void_p, _c_ll, _c_void_p, _c_void_p]),
+    "csrspmm_csr_i64_to_i32": (_c_int, [_c_void_p, _c_void_p, _c_ll, _c_void_p, _c_void_p, _c_ll,
+                                        _c_void_p]),
     "csrspmm_device_malloc": (_c_int, [ctypes.POINTER(_c_void_p), _c_size_t]),
     "csrspmm_device_free": (_c_int, [_c_void_p]),
     "csrspmm_memcpy_h2d": (_c_int, [_c_void_p, _c_void_p, _c_size_t]),

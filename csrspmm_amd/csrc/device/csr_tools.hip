@@ -377,6 +377,21 @@ __global__ __launch_bounds__(kToolBlock) void narrow_kernel(const long long* src
   if (overflow && __ballot(bad) && lane_id() == 0) *overflow = 1;
 }
 
+// dst0[i] = src0[i] for i < n0 and dst1[i] = src1[i] for i < n1, the low 32 bits:
+// both index arrays of a CSR in one launch (2^21 entries: 2 x 5.2 us before).
+__global__ __launch_bounds__(kToolBlock) void narrow_csr_kernel(const long long* src0, int* dst0, long long n0,
+                                                                const long long* src1, int* dst1,
+                                                                long long n1) {
+  for (long long i = (long long)blockIdx.x * blockDim.x + threadIdx.x; i < n0 + n1;
+       i += (long long)gridDim.x * blockDim.x) {
+    if (i < n0) {
+      dst0[i] = static_cast<int>(src0[i]);
+    } else {
+      dst1[i - n0] = static_cast<int>(src1[i - n0]);
+    }
+  }
+}
+
 int tool_blocks(long long work, int per_block) {
   return static_cast<int>(std::max<long long>(1, std::min<long long>(kToolMaxBlocks, (work + per_block - 1) / per_block)));
 }
@@ -477,6 +492,19 @@ int csrspmm_indices_i64_to_i32(const long long* src, int* dst, long long n, int*
   if (n > 0)
     hipLaunchKernelGGL(narrow_kernel, dim3(tool_blocks(n, kToolBlock)), dim3(kToolBlock), 0, s, src,
                        dst, n, overflow_out);
+  return status_of(hipGetLastError());
+}
+
+int csrspmm_csr_i64_to_i32(const long long* rowptr, int* rowptr_out, long long n_rowptr, const long long* colidx,
+                           int* colidx_out, long long n_colidx, void* stream) {
+  if (n_rowptr < 0 || n_colidx < 0 || (n_rowptr > 0 && (!rowptr || !rowptr_out)) ||
+      (n_colidx > 0 && (!colidx || !colidx_out)))
+    return CSRSPMM_STATUS_INVALID_VALUE;
+  if (n_rowptr + n_colidx == 0) return CSRSPMM_STATUS_SUCCESS;
+  hipStream_t s = static_cast<hipStream_t>(stream);
+  (void)hipGetLastError();
+  hipLaunchKernelGGL(narrow_csr_kernel, dim3(tool_blocks(n_rowptr + n_colidx, kToolBlock)), dim3(kToolBlock), 0, s,
+                     rowptr, rowptr_out, n_rowptr, colidx, colidx_out, n_colidx);
   return status_of(hipGetLastError());
 }
 

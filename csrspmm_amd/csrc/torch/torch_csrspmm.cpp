@@ -339,10 +339,42 @@ Tensor indices_to_int32(Tensor idx) {
   return dst;
 }
 
+// The forwards' semantics (new C, beta scaling zero) for a torch.sparse_csr A:
+// int32 indices in place, int64 ones narrowed by one launch (A's sizes fit
+// int32, which makes that exact for a valid CSR).
+Tensor csrspmm_sparse(Tensor A, Tensor B, double alpha, double beta, const std::string& algo) {
+  TORCH_CHECK(A.layout() == at::kSparseCsr, "A must be a torch.sparse_csr tensor");
+  TORCH_CHECK(A.is_cuda(), "A must be a CUDA tensor");
+  TORCH_CHECK(A.dim() == 2, "A must be 2-D (no batch dimensions)");
+  const int64_t M = A.size(0), K = A.size(1);
+  Tensor vals = A.values();
+  TORCH_CHECK(M < INT32_MAX && K <= INT32_MAX && vals.numel() <= INT32_MAX, "A's sizes must fit int32");
+  TORCH_CHECK(vals.dtype() == torch::kFloat32, "A_values must be float32");
+  Tensor rowptr = A.crow_indices().contiguous(), colidx = A.col_indices().contiguous();
+  TORCH_CHECK(B.dim() == 2 && B.size(0) == K, "B must be [K, N] with K = A.shape[1]");
+  if (rowptr.dtype() == torch::kInt64 && colidx.dtype() == torch::kInt64) {
+    c10::DeviceGuard guard(A.device());
+    Tensor r32 = torch::empty({rowptr.size(0)}, rowptr.options().dtype(torch::kInt32));
+    Tensor c32 = torch::empty({colidx.size(0)}, colidx.options().dtype(torch::kInt32));
+    const int st = csrspmm_csr_i64_to_i32(
+        reinterpret_cast<const long long*>(rowptr.data_ptr<int64_t>()), r32.data_ptr<int>(), rowptr.size(0),
+        reinterpret_cast<const long long*>(colidx.numel() ? colidx.data_ptr<int64_t>() : nullptr),
+        colidx.numel() ? c32.data_ptr<int>() : nullptr, colidx.size(0), stream_of(rowptr));
+    TORCH_CHECK(st == 0, "csrspmm_sparse failed: ", csrspmm_status_string(st));
+    rowptr = r32;
+    colidx = c32;
+  } else {
+    rowptr = indices_to_int32(rowptr);
+    colidx = indices_to_int32(colidx);
+  }
+  return forward(algo_id(algo), rowptr, colidx, vals.contiguous(), -1, B, alpha, beta);
+}
+
 }  // namespace
 
 PYBIND11_MODULE(TORCH_EXTENSION_NAME, m) {
   m.def("csrspmm_forward", &csrspmm_forward_named, "CSR SpMM by variant name (new C)");
+  m.def("csrspmm_sparse", &csrspmm_sparse, "CSR SpMM of a torch.sparse_csr tensor (new C)");
   m.def("dense_to_csr", &dense_to_csr, "device dense -> CSR (rowptr, colidx, values)");
   m.def("csr_max_row_nnz", &csr_max_row_nnz, "longest row, on the device");
   m.def("indices_to_int32", &indices_to_int32, "int64 -> int32 CSR indices, on the device");

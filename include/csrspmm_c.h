@@ -371,6 +371,12 @@ int csrspmm_csr_max_row_nnz(int M, const int* rowptr, int* max_out, void* stream
 int csrspmm_indices_i64_to_i32(const long long* src, int* dst, long long n, int* overflow_out,
                                void* stream);
 
+/* Both index arrays of a CSR narrowed so in one launch, for arrays whose values
+ * are known to fit (a valid CSR whose nnz and K do). */
+int csrspmm_csr_i64_to_i32(const long long* rowptr, int* rowptr_out, long long n_rowptr,
+                           const long long* colidx, int* colidx_out, long long n_colidx,
+                           void* stream);
+
 /* Memory and device helpers that let the g++-built C++ layer stay free of
  * HIP headers (they back csr_alloc_device / dense_alloc_device and the
  * host<->device copies at reference src/host/csr_utils.cpp:44-67,183-238 and

@@ -129,10 +129,7 @@ def from_sparse_csr(A):
 def csrspmm_sparse(A, B, alpha=1.0, beta=0.0, algo="Auto"):
     """C = alpha * A @ B for a torch.sparse_csr A (a new C; beta scales a zero
     C, as in the five entry points)."""
-    rowptr, colidx, vals, K = from_sparse_csr(A)
-    if B.dim() != 2 or B.size(0) != K:
-        raise RuntimeError("B must be [K, N] with K = A.shape[1]")
-    return _C.csrspmm_forward(rowptr, colidx, vals, B, alpha, beta, algo)
+    return _C.csrspmm_sparse(A, B, alpha, beta, algo)
 
 
 def dense_to_csr(D, tol=0.0):
