@@ -275,6 +275,21 @@ __global__ __launch_bounds__(256) void naive_smem_kernel(Problem p, int ntile, i
   }
 }
 
+// Unused LDS that leaves room for 5 blocks (20 waves) a CU instead of 8, for
+// rows that average kNaiveCapMean nonzeros or more on a B beyond kNaiveCapBytes:
+// their batches of 32 gathers, cheap as they are to issue, push each other's
+// B rows out of the L2s.  Measured on MI355X per call, 8 blocks -> 6 -> 5:
+// 65536^2 x 256 with 66 per row 504 -> 498 -> 486 us, with 0-200 (60000^2) 681
+// -> 667 -> 650, 131072^2 x 128 with 40 352 -> 349 -> 339; but with 30 per row
+// 237 -> 258 -> 309, and the relays of skewed rows (mean 16) 75 -> 88 -> 115.
+constexpr int kNaiveCapMean = 36;
+constexpr long long kNaiveCapBytes = 32LL << 20;
+constexpr int kNaiveCapBlocks = 5;
+inline unsigned naive_pad_lds(const Problem& p) {
+  if (p.nnz < (long long)kNaiveCapMean * p.M || (long long)p.K * p.N * 4 <= kNaiveCapBytes) return 0;
+  return (unsigned)(kLdsPerCu / kNaiveCapBlocks / 512 * 512 - 1024);  // the static sums take 512
+}
+
 }  // namespace
 
 hipError_t launch_naive(const Problem& p, hipStream_t s) {
@@ -285,13 +300,14 @@ hipError_t launch_naive(const Problem& p, hipStream_t s) {
   const long long blocks = ((long long)div_up_host(p.M, kNaiveWaves) + long_blocks) * ntile;
   if (blocks > 0x7fffffffLL) return hipErrorInvalidValue;
   timing_before_main(s);
+  const unsigned pad_lds = naive_pad_lds(p);
   const bool buf = p.K > 0 && (long long)(p.K - 1) * p.ldb * 4 + (long long)p.N * 4 < (1LL << 32);
   if (buf) {
-    hipLaunchKernelGGL((naive_kernel<true>), dim3((unsigned)blocks), dim3(kNaiveWaves * 64), 0, s, p, ntile,
-                       long_blocks, long_row);
+    hipLaunchKernelGGL((naive_kernel<true>), dim3((unsigned)blocks), dim3(kNaiveWaves * 64), pad_lds, s, p,
+                       ntile, long_blocks, long_row);
   } else {
-    hipLaunchKernelGGL((naive_kernel<false>), dim3((unsigned)blocks), dim3(kNaiveWaves * 64), 0, s, p, ntile,
-                       long_blocks, long_row);
+    hipLaunchKernelGGL((naive_kernel<false>), dim3((unsigned)blocks), dim3(kNaiveWaves * 64), pad_lds, s, p,
+                       ntile, long_blocks, long_row);
   }
   const hipError_t e = hipGetLastError();
   timing_after_main(s);

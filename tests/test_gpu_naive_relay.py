@@ -54,6 +54,17 @@ def test_one_block_relays_many_rows(gpu):
     assert np.array_equal(C, oracle.spmm_f32_seq(rp, ci, va, B, None, 1.0, 0.0))
 
 
+@pytest.mark.parametrize("per_row", [35, 36, 600])
+def test_fewer_blocks_on_a_large_b(per_row, gpu):
+    """B just above 32 MiB around 36 nonzeros a row (blocks a CU are capped from
+    there), without and with relayed rows."""
+    M, K, N = 301, 70001, 120
+    rp, ci, va = csr_from_lengths(np.full(M, per_row), K, seed=per_row)
+    B = np.random.default_rng(9).uniform(-1, 1, (K, N)).astype(np.float32)
+    C = tc.csrspmm_naive(t(rp, gpu), t(ci, gpu), t(va, gpu), t(B, gpu), 1.0, 0.0).cpu().numpy()
+    assert np.array_equal(C, oracle.spmm_f32_seq(rp, ci, va, B, None, 1.0, 0.0))
+
+
 def test_b_beyond_4_gib(gpu):
     """64-bit row addresses: a view of 70 columns of rows 2^17 floats apart."""
     K, N, ld = 9000, 70, 1 << 17
